@@ -1,4 +1,5 @@
-// fp32 GEMM family on CDNA4 matrix cores (v_mfma_f32_16x16x4_f32) for the reference's
+// fp32 GEMM family on CDNA4 matrix cores (v_mfma_f32_16x16x4_f32; larger products on bf16 planes,
+// gemm_split.hip) for the reference's
 // matmul / matmul_left_backward / matmul_right_backward (runtime/backend.rs:934-1021,
 // kernels :2190-2290), and implicit-GEMM convolution entries that compute the reference's
 // unfold -> contract (forward), contract-backward -> unfold_backward (dgrad) and
@@ -39,11 +40,13 @@
 #include "conv_small.hpp"
 #include "fastdiv.hpp"
 #include "gemm_bf16.hpp"
-#include "pool_rule.hpp"
+#include "gemm_parts.hpp"
+#include "gemm_split.hpp"
 
 namespace {
 
-typedef float floatx4 __attribute__((ext_vector_type(4)));
+using namespace axis;
+
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 // Split partial sums of the allocation-free weight gradient (axis_matmul_right_backward_noalloc).
@@ -60,114 +63,6 @@ struct Workspace {
     float *ptr;
     int64_t floats;
 };
-
-// Geometry of a gathered convolution operand (tensor [batch, height, width, channels]).
-struct ConvGeom {
-    const float *src;
-    int64_t ld_b;                     // element strides of batch, channel, row, column
-    int32_t ld_c, ld_h, ld_w;
-    int32_t height, width, channels;  // gathered tensor
-    int32_t out_h, out_w;             // output pixel grid the reduction/rows enumerate
-    int32_t kh, kw, sy, sx, py, px;
-    FastDiv c_div, kw_div, ow_div, oh_div;
-    bool tap_steps;                   // channels % 32 == 0: a 32-deep K step stays in one tap
-    // With tap steps, the buffer rows loader walks the reduction in 32-channel blocks, every tap
-    // of a block before the next block: r = (cb * taps + pos) * 32 + ci.  A tile then re-reads
-    // the same 32 channels of its neighbourhood on consecutive steps, which stay in L2, instead
-    // of the whole tensor slab between one tap and the next.
-    bool block_major;
-    FastDiv taps_div;                 // kh * kw
-    // Rows mode, 2x2 pooling epilogue: tile row t holds position t % 4 (ky major) of the tile's
-    // window t / 4, windows numbered row-major over the tile's window rows (pw per row).  A tile
-    // starts on an even output row and holds whole window rows.
-    bool window_major;
-    FastDiv pw_div;
-};
-
-// Output pixel of tile row t for a tile starting at pixel t0.
-__device__ __forceinline__ int64_t tile_pixel(const ConvGeom &g, int64_t t0, int t) {
-    if (!g.window_major) return t0 + t;
-    const uint32_t w = (uint32_t)t >> 2, pos = (uint32_t)t & 3u;
-    const uint32_t wr = g.pw_div.div(w), wc = w - wr * g.pw_div.d;
-    return t0 + (int64_t)(2 * wr + (pos >> 1)) * g.out_w + 2 * wc + (pos & 1u);
-}
-
-// Second operand read straight from a convolution weight in the reference's [(c, ky, kx), n]
-// layout: the reduction index is r = pos * R + q (pos = ky * kw + kx, R rows per tap, R a
-// multiple of the K step), and a K step starting at r0 = pos * R + q0 begins at element
-// q0 * qa + pos * pb + pc, its rows s_r apart.
-struct TapSteps {
-    bool on;
-    FastDiv r_div;   // R
-    int64_t qa, pb, pc;
-    // The rows loader's block-major order: step r0 = (cb * taps + pos) * 32 covers q0 = 32 cb.
-    bool block_major;
-    FastDiv taps_div;
-};
-
-struct GemmParams {
-    const float *x;
-    const float *y;
-    float *c;
-    const float *bias;         // added to every row of C (length n), or null
-    const float *d;            // out = beta * d + alpha * (A.B) when non-null (d shaped like out)
-    float alpha, beta;
-    int64_t m, n, k;           // C is [m, n]; reduction length k
-    int64_t x_si, x_sr;        // dense X(i, r) = x[i * x_si + r * x_sr]
-    int64_t y_sr, y_sj;        // Y(r, j) = y[r * y_sr + j * y_sj]
-    int64_t x_batch, y_batch;  // batch strides (elements)
-    int64_t c_batch;           // batch stride of the output (or of one slice of partials)
-    int64_t c_split;           // stride between reduction slices in the output (partials)
-    int64_t k_chunk;           // reduction length per slice (multiple of the tile depth)
-    int64_t k_work;            // algorithmic reduction length for timing (k without padding), or 0
-    int32_t splits;
-    int32_t tiles_m, tiles_n;
-    uint32_t xcd_span;         // blocks / 8: the first 8 * xcd_span blocks are remapped, the rest keep their order
-    ConvGeom conv;
-    // Pooling epilogue: output rows are pixels of a [.., out_h, out_w] grid (out_w = pool_ow).
-    float *pooled;
-    uint8_t *argmax;
-    int32_t pool_h, pool_w, pool_ow;
-    FastDiv pool_cols;         // pooled columns per output row (pool_ow / pool_w)
-    TapSteps ytaps;            // Y read as a tap-major convolution weight
-    // Output rows ordered (pos, c) with perm_c channels and perm_taps taps are written as rows
-    // c * perm_taps + pos (the reference's weight layout); 0 = rows as computed.
-    int32_t perm_c, perm_taps;
-    bool bf16;                 // operands rounded to bf16 as they are staged (Device::cuda_bf16)
-};
-
-template <int VEC>
-__device__ __forceinline__ void load_into(float *reg, const float *src, bool valid) {
-    if constexpr (VEC == 4) {
-        floatx4 v = {0.f, 0.f, 0.f, 0.f};
-        if (valid) v = *reinterpret_cast<const floatx4 *>(src);
-        reg[0] = v[0];
-        reg[1] = v[1];
-        reg[2] = v[2];
-        reg[3] = v[3];
-    } else {
-        reg[0] = valid ? src[0] : 0.f;
-    }
-}
-
-// Buffer loads: an offset at or past the resource's record count (2^31 - 1 bytes) reads as zero,
-// so padding taps and reduction tails need neither a branch nor zeroed registers.
-constexpr uint32_t kOutside = 0x80000000u;
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const float *base, int32_t bytes = 0x7fffffff) {
-    return __builtin_amdgcn_make_buffer_rsrc((void *)base, (short)0, bytes, 0x00020000);
-}
-template <int VEC>
-__device__ __forceinline__ void buffer_into(float *reg, __amdgpu_buffer_rsrc_t rsrc, uint32_t byte_offset) {
-    if constexpr (VEC == 4) {
-        const floatx4 v = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, byte_offset, 0, 0));
-        reg[0] = v[0];
-        reg[1] = v[1];
-        reg[2] = v[2];
-        reg[3] = v[3];
-    } else {
-        reg[0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, byte_offset, 0, 0));
-    }
-}
 
 // LDS staging shared by every loader: [r][t] layout, row pitch BT + 4 (16-byte aligned rows),
 // and column t of row r stored at t ^ swizzle(r) with swizzle(r) = 8 * ((r / 4) % 8).  The XOR
@@ -194,6 +89,10 @@ struct Staging {
     static constexpr int LD = RCONTIG && BT >= 64 ? BT + 64 : BT + 4;
     static constexpr int kPer = RCONTIG ? BK / VEC : BT / VEC;  // vectors per contiguous line
     float reg[kElems];
+    static __device__ __forceinline__ int line_r(int idx) { return (idx % kPer) * VEC; }  // NT is a multiple of kPer
+    static __device__ __forceinline__ int line_t(int idx) { return idx / kPer; }
+    static __device__ __forceinline__ int vec_t(int tid) { return (tid % kPer) * VEC; }
+    static __device__ __forceinline__ int vec_r(int tid, int e) { return tid / kPer + e * (NT / kPer); }
 
     // bf16: round every staged operand to bf16 first (products of bf16 values are exact in fp32).
     __device__ __forceinline__ void store(float *__restrict__ lds, int tid, int bf16 = 0) {
@@ -222,15 +121,6 @@ struct Staging {
         }
     }
 };
-
-// A wave-uniform pointer moved to scalar registers, so that buffer resources built from it need no
-// per-lane loop (the compiler cannot always prove such values uniform).
-__device__ __forceinline__ const float *uniform_ptr(const float *p) {
-    const uint64_t v = reinterpret_cast<uint64_t>(p);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return reinterpret_cast<const float *>(((uint64_t)hi << 32) | lo);
-}
 
 // Dense operand: element (t, r) at base[t * s_t + r * s_r], read through buffer loads.  One buffer
 // resource per K step, based at the tile's element (t0, step) (wave-uniform: a 64-bit scalar add and
@@ -279,20 +169,7 @@ struct DenseLoader : Staging<BT, BK, NT, RCONTIG, VEC> {
     template <bool WHOLE = false>
     __device__ __forceinline__ void load(const ConvGeom &, int64_t r0, int32_t room, int) {
         int64_t step = r0 * s_r;
-        if (taps.on) {
-            uint32_t pos;
-            int64_t q0;
-            if (taps.block_major) {
-                const uint32_t st = (uint32_t)r0 >> 5;
-                const uint32_t cb = taps.taps_div.div(st);
-                pos = st - cb * taps.taps_div.d;
-                q0 = (int64_t)cb * 32;
-            } else {
-                pos = taps.r_div.div((uint32_t)r0);
-                q0 = r0 - (int64_t)pos * taps.r_div.d;
-            }
-            step = q0 * taps.qa + (int64_t)pos * taps.pb + taps.pc;
-        }
+        if (taps.on) step = taps.step(r0);
         if constexpr (RCONTIG) {
             const __amdgpu_buffer_rsrc_t rsrc = make_rsrc(uniform_ptr(tile_base + step));
             // Branch-free: split into whole-step and partial-step paths, the loads' wait counts
@@ -310,277 +187,6 @@ struct DenseLoader : Staging<BT, BK, NT, RCONTIG, VEC> {
 #pragma unroll
             for (int e = 0; e < S::kVecs; ++e) buffer_into<VEC>(this->reg + e * VEC, rsrc, voff[e]);
         }
-    }
-};
-
-// Convolution operand, rows mode: t = output pixel, r = (ky*kw + kx)*channels + channel.
-// Per row: the offset of its window origin and the origin's coordinates (for the padding test);
-// per K step: one decode of the thread's r into a 32-bit offset shared by every row.
-template <int BT, int BK, int NT, int VEC>
-struct ConvRowsLoader : Staging<BT, BK, NT, true, VEC> {
-    using S = Staging<BT, BK, NT, true, VEC>;
-    uint32_t origin[S::kVecs];   // b*ld_b + iy0*ld_h + ix0*ld_w (mod 2^32; exact when valid)
-    int32_t iy0[S::kVecs], ix0[S::kVecs];
-    int rr;
-
-    __device__ __forceinline__ void init(const ConvGeom &geom, int64_t t0, int64_t t_end, int tid) {
-        rr = (tid % S::kPer) * VEC;  // NT is a multiple of kPer, so rr is the same for every e
-#pragma unroll
-        for (int e = 0; e < S::kVecs; ++e) {
-            const int64_t gt = tile_pixel(geom, t0, (tid + e * NT) / S::kPer);
-            // Rows past the end get an origin far outside the image, so every tap is padding;
-            // computed branch-free so the per-row arrays stay in registers.
-            const bool live = gt < t_end;
-            const uint32_t pix = live ? (uint32_t)gt : 0u;
-            const uint32_t q = geom.ow_div.div(pix);
-            const int32_t ox = (int32_t)(pix - q * (uint32_t)geom.out_w);
-            const uint32_t b = geom.oh_div.div(q);
-            const int32_t oy = (int32_t)(q - b * (uint32_t)geom.out_h);
-            const int32_t y0 = oy * geom.sy - geom.py;
-            ix0[e] = ox * geom.sx - geom.px;
-            origin[e] = b * (uint32_t)geom.ld_b + (uint32_t)y0 * (uint32_t)geom.ld_h +
-                        (uint32_t)ix0[e] * (uint32_t)geom.ld_w;
-            iy0[e] = live ? y0 : -(1 << 30);
-        }
-    }
-    __device__ __forceinline__ void load(const ConvGeom &geom, int64_t r0, int32_t room, int) {
-        const bool r_ok = rr < room;
-        const uint32_t g = r_ok ? (uint32_t)(r0 + rr) : 0u;
-        const uint32_t pos = geom.c_div.div(g);
-        const int32_t c = (int32_t)(g - pos * (uint32_t)geom.channels);
-        const int32_t ky = (int32_t)geom.kw_div.div(pos);
-        const int32_t kx = (int32_t)pos - ky * geom.kw;
-        const uint32_t delta = (uint32_t)(ky * geom.ld_h + kx * geom.ld_w + c * geom.ld_c);
-#pragma unroll
-        for (int e = 0; e < S::kVecs; ++e) {
-            const bool valid = r_ok && (uint32_t)(iy0[e] + ky) < (uint32_t)geom.height &&
-                               (uint32_t)(ix0[e] + kx) < (uint32_t)geom.width;
-            load_into<VEC>(this->reg + e * VEC, geom.src + (valid ? origin[e] + delta : 0u), valid);
-        }
-    }
-};
-
-// Rows mode through buffer loads, for gathered tensors whose offsets fit 31-bit byte offsets and
-// kernels of at most 32 taps.  Each row keeps its window origin's offset and a mask of the taps
-// that fall outside the image (bit ky*kw + kx), so a K step tests one bit per vector.  When the
-// channel count is a multiple of BK (geom.tap_steps), a K step covers BK channels of one tap and
-// the step's tap decode is wave-uniform.
-template <int BT, int BK, int NT, int VEC>
-struct ConvRowsBufferLoader : Staging<BT, BK, NT, true, VEC> {
-    using S = Staging<BT, BK, NT, true, VEC>;
-    uint32_t origin4[S::kVecs];  // 4 * (b*ld_b + iy0*ld_h + ix0*ld_w) (mod 2^32; exact when valid)
-    uint32_t outside[S::kVecs];  // taps of the row's window outside the image (all, for rows past the end)
-    int rr;
-    uint32_t lane_c4;            // 4 * rr * ld_c: the thread's channel offset inside a tap step, bytes
-
-    __device__ __forceinline__ void init(const ConvGeom &geom, int64_t t0, int64_t t_end, int tid) {
-        rr = (tid % S::kPer) * VEC;
-        lane_c4 = (uint32_t)(rr * geom.ld_c) * 4u;
-#pragma unroll
-        for (int e = 0; e < S::kVecs; ++e) {
-            const int64_t gt = tile_pixel(geom, t0, (tid + e * NT) / S::kPer);
-            const bool live = gt < t_end;
-            const uint32_t pix = live ? (uint32_t)gt : 0u;
-            const uint32_t q = geom.ow_div.div(pix);
-            const int32_t ox = (int32_t)(pix - q * (uint32_t)geom.out_w);
-            const uint32_t b = geom.oh_div.div(q);
-            const int32_t oy = (int32_t)(q - b * (uint32_t)geom.out_h);
-            const int32_t y0 = oy * geom.sy - geom.py;
-            const int32_t x0 = ox * geom.sx - geom.px;
-            origin4[e] = (b * (uint32_t)geom.ld_b + (uint32_t)y0 * (uint32_t)geom.ld_h + (uint32_t)x0 * (uint32_t)geom.ld_w) * 4u;
-            uint32_t cols = 0, taps = 0;
-            for (int32_t kx = 0; kx < geom.kw; ++kx)
-                cols |= (uint32_t)((uint32_t)(x0 + kx) < (uint32_t)geom.width) << kx;
-            for (int32_t ky = 0; ky < geom.kh; ++ky)
-                taps |= ((uint32_t)(y0 + ky) < (uint32_t)geom.height ? cols : 0u) << (ky * geom.kw);
-            outside[e] = live ? ~taps : ~0u;
-        }
-    }
-    __device__ __forceinline__ void load(const ConvGeom &geom, int64_t r0, int32_t room, int) {
-        const __amdgpu_buffer_rsrc_t rsrc = make_rsrc(geom.src);
-        if (geom.tap_steps) {
-            // The reduction is a multiple of BK here, so every k of the step is inside it; the
-            // step's tap and first channel are wave-uniform (scalar arithmetic).  Per vector: the
-            // offset, and the window's outside bit for this tap moved to bit 31, which puts a
-            // masked lane's offset past the record count (three vector instructions).
-            uint32_t pos;
-            int32_t c0;
-            if (geom.block_major) {
-                const uint32_t st = (uint32_t)r0 >> 5;
-                const uint32_t cb = geom.taps_div.div(st);
-                pos = st - cb * geom.taps_div.d;
-                c0 = (int32_t)cb * 32;
-            } else {
-                pos = geom.c_div.div((uint32_t)r0);
-                c0 = (int32_t)((uint32_t)r0 - pos * (uint32_t)geom.channels);
-            }
-            const int32_t ky = (int32_t)geom.kw_div.div(pos);
-            const int32_t kx = (int32_t)pos - ky * geom.kw;
-            const uint32_t delta4 =
-                __builtin_amdgcn_readfirstlane((uint32_t)(ky * geom.ld_h + kx * geom.ld_w + c0 * geom.ld_c) * 4u) +
-                lane_c4;
-            const uint32_t up = 31u - __builtin_amdgcn_readfirstlane(pos);
-#pragma unroll
-            for (int e = 0; e < S::kVecs; ++e)
-                buffer_into<VEC>(this->reg + e * VEC, rsrc, (origin4[e] + delta4) | ((outside[e] << up) & kOutside));
-        } else {
-            const bool r_ok = rr < room;
-            const uint32_t g = r_ok ? (uint32_t)(r0 + rr) : 0u;
-            const uint32_t pos = geom.c_div.div(g);
-            const int32_t c = (int32_t)(g - pos * (uint32_t)geom.channels);
-            const int32_t ky = (int32_t)geom.kw_div.div(pos);
-            const int32_t kx = (int32_t)pos - ky * geom.kw;
-            const uint32_t delta4 = (uint32_t)(ky * geom.ld_h + kx * geom.ld_w + c * geom.ld_c) * 4u;
-#pragma unroll
-            for (int e = 0; e < S::kVecs; ++e) {
-                const bool valid = r_ok && ((outside[e] >> pos) & 1u) == 0;
-                buffer_into<VEC>(this->reg + e * VEC, rsrc, valid ? origin4[e] + delta4 : kOutside);
-            }
-        }
-    }
-};
-
-// Convolution operand, cols mode: t = (ky*kw + kx)*channels + channel, r = output pixel.  The
-// thread's t is fixed; each row keeps its pixel's coordinates and offset and walks forward BK
-// pixels per K step.
-template <int BT, int BK, int NT, int VEC>
-struct ConvColsLoader : Staging<BT, BK, NT, false, VEC> {
-    using S = Staging<BT, BK, NT, false, VEC>;
-    static constexpr int kRowStep = NT / S::kPer;  // pixels between the thread's rows
-    uint32_t tap;                // (ky-py)*ld_h + (kx-px)*ld_w + c*ld_c of the thread's t (mod 2^32)
-    int32_t ky, kx;
-    bool t_ok;
-    int32_t ox[S::kVecs], oy[S::kVecs];
-    uint32_t off[S::kVecs];      // b*ld_b + oy*sy*ld_h + ox*sx*ld_w (mod 2^32)
-    int64_t next_r;              // r0 the state describes
-
-    __device__ __forceinline__ void init(const ConvGeom &geom, int64_t t0, int64_t t_end, int tid) {
-        const int64_t gt = t0 + (tid % S::kPer) * VEC;
-        t_ok = gt < t_end;
-        const uint32_t g = t_ok ? (uint32_t)gt : 0u;
-        const uint32_t pos = geom.c_div.div(g);
-        const int32_t c = (int32_t)(g - pos * (uint32_t)geom.channels);
-        ky = (int32_t)geom.kw_div.div(pos);
-        kx = (int32_t)pos - ky * geom.kw;
-        tap = (uint32_t)(ky - geom.py) * (uint32_t)geom.ld_h + (uint32_t)(kx - geom.px) * (uint32_t)geom.ld_w +
-              (uint32_t)c * (uint32_t)geom.ld_c;
-        next_r = -1;
-    }
-    __device__ __forceinline__ void locate(const ConvGeom &geom, int64_t r0, int tid) {
-#pragma unroll
-        for (int e = 0; e < S::kVecs; ++e) {
-            const uint32_t pix = (uint32_t)(r0 + tid / S::kPer + e * kRowStep);
-            const uint32_t q = geom.ow_div.div(pix);
-            ox[e] = (int32_t)(pix - q * (uint32_t)geom.out_w);
-            const uint32_t b = geom.oh_div.div(q);
-            oy[e] = (int32_t)(q - b * (uint32_t)geom.out_h);
-            off[e] = b * (uint32_t)geom.ld_b + (uint32_t)(oy[e] * geom.sy) * (uint32_t)geom.ld_h +
-                     (uint32_t)(ox[e] * geom.sx) * (uint32_t)geom.ld_w;
-        }
-        next_r = r0;
-    }
-    __device__ __forceinline__ void advance(const ConvGeom &geom) {
-        const uint32_t col_step = (uint32_t)(geom.sx * geom.ld_w), row_step = (uint32_t)(geom.sy * geom.ld_h);
-#pragma unroll
-        for (int e = 0; e < S::kVecs; ++e) {
-            ox[e] += BK;
-            off[e] += BK * col_step;
-            while (ox[e] >= geom.out_w) {
-                ox[e] -= geom.out_w;
-                off[e] += row_step - (uint32_t)geom.out_w * col_step;
-                if (++oy[e] == geom.out_h) {
-                    oy[e] = 0;
-                    off[e] += (uint32_t)geom.ld_b - (uint32_t)geom.out_h * row_step;
-                }
-            }
-        }
-        next_r += BK;
-    }
-    __device__ __forceinline__ void load(const ConvGeom &geom, int64_t r0, int32_t room, int tid) {
-        if (r0 != next_r) locate(geom, r0, tid);
-#pragma unroll
-        for (int e = 0; e < S::kVecs; ++e) {
-            const int32_t iy = oy[e] * geom.sy + ky - geom.py, ix = ox[e] * geom.sx + kx - geom.px;
-            const bool valid = t_ok && tid / S::kPer + e * kRowStep < room && (uint32_t)iy < (uint32_t)geom.height &&
-                               (uint32_t)ix < (uint32_t)geom.width;
-            load_into<VEC>(this->reg + e * VEC, geom.src + (valid ? off[e] + tap : 0u), valid);
-        }
-        advance(geom);
-    }
-};
-
-// Cols mode when every K step covers whole aligned pixel runs: BK divides the output width or is
-// a multiple of it, and the image's pixel count is a multiple of BK.  Then a step starting at
-// pixel p0 (a multiple of BK) never leaves one image and the in-step pixel s sits at
-// (oy0 + s / out_w, ox0 + s % out_w) for every step, so each vector's window position relative
-// to the step origin is fixed at init and a step decodes only its wave-uniform origin.
-template <int BT, int BK, int NT, int VEC>
-struct ConvColsStepLoader : Staging<BT, BK, NT, false, VEC> {
-    using S = Staging<BT, BK, NT, false, VEC>;
-    static constexpr int kRowStep = NT / S::kPer;  // pixels between the thread's rows
-    static_assert(BK == 32, "steps of 32 pixels");
-    uint32_t rel4[S::kVecs];  // bytes: (iy_rel + py)*ld_h + (ix_rel + px)*ld_w + c*ld_c (mod 2^32)
-    // Bit (first | last << 1 | top << 2 | bottom << 3) set when the lane's element is padding (or
-    // its row past the end) in a step whose pixels start the image's first / last 32-column
-    // segment, first / last row group.  A step elsewhere has every element inside (the host
-    // keeps px <= 32 sx and py <= (rows per step) sy), so these four flags decide.
-    uint32_t bad[S::kVecs];
-
-    __device__ __forceinline__ void init(const ConvGeom &geom, int64_t t0, int64_t t_end, int tid) {
-        const int64_t gt = t0 + (tid % S::kPer) * VEC;
-        const bool t_ok = gt < t_end;
-        const uint32_t g = t_ok ? (uint32_t)gt : 0u;
-        const uint32_t pos = geom.c_div.div(g);
-        const int32_t c = (int32_t)(g - pos * (uint32_t)geom.channels);
-        const int32_t ky = (int32_t)geom.kw_div.div(pos);
-        const int32_t kx = (int32_t)pos - ky * geom.kw;
-        const int32_t s0 = tid / S::kPer;
-        const int32_t seg = geom.out_w < 32 ? geom.out_w : 32;       // columns a step spans
-        const int32_t rows = geom.out_w < 32 ? 32 / geom.out_w : 1;  // rows a step spans
-        const int32_t last_x = (geom.out_w - seg) * geom.sx, last_y = (geom.out_h - rows) * geom.sy;
-#pragma unroll
-        for (int e = 0; e < S::kVecs; ++e) {
-            const uint32_t s = (uint32_t)(s0 + e * kRowStep);
-            const int32_t dy = (int32_t)geom.ow_div.div(s);
-            const int32_t dx = (int32_t)s - dy * geom.out_w;
-            const int32_t iy_rel = dy * geom.sy + ky - geom.py, ix_rel = dx * geom.sx + kx - geom.px;
-            rel4[e] = ((uint32_t)(iy_rel + geom.py) * (uint32_t)geom.ld_h + (uint32_t)(ix_rel + geom.px) * (uint32_t)geom.ld_w +
-                       (uint32_t)c * (uint32_t)geom.ld_c) * 4u;
-            uint32_t b = 0;
-            for (uint32_t f = 0; f < 16; ++f) {
-                const bool first = f & 1u, last = f & 2u, top = f & 4u, bottom = f & 8u;
-                const int32_t x = first ? ix_rel : last ? last_x + ix_rel : 0;
-                const int32_t y = top ? iy_rel : bottom ? last_y + iy_rel : 0;
-                const bool in = t_ok && (!(first || last) || (uint32_t)x < (uint32_t)geom.width) &&
-                                (!(top || bottom) || (uint32_t)y < (uint32_t)geom.height);
-                b |= (in ? 0u : 1u) << f;
-            }
-            bad[e] = b;
-        }
-    }
-    // Every step is whole: the reduction (batch * image pixels) and the slices are multiples of 32.
-    __device__ __forceinline__ void load(const ConvGeom &geom, int64_t r0, int32_t, int) {
-        const uint32_t p0 = (uint32_t)r0;
-        const uint32_t q = geom.ow_div.div(p0);
-        const int32_t ox0 = (int32_t)(p0 - q * (uint32_t)geom.out_w);
-        const uint32_t b = geom.oh_div.div(q);
-        const int32_t oy0 = (int32_t)(q - b * (uint32_t)geom.out_h);
-        const int32_t seg = geom.out_w < 32 ? geom.out_w : 32;
-        const int32_t rows = geom.out_w < 32 ? 32 / geom.out_w : 1;
-        // sign bits rather than comparisons: compared flags reach vector registers as lane masks
-        const uint32_t flags = ((uint32_t)(ox0 - 1) >> 31) | ((uint32_t)(geom.out_w - ox0 - seg - 1) >> 31 << 1) |
-                               ((uint32_t)(oy0 - 1) >> 31 << 2) | ((uint32_t)(geom.out_h - oy0 - rows - 1) >> 31 << 3);
-        const int32_t oys = oy0 * geom.sy, oxs = ox0 * geom.sx;
-        // Buffer base at the step origin moved back by the padding, so that every valid lane's
-        // offset (at least -py rows and -px columns from the origin) is non-negative.
-        const int64_t shift = (int64_t)geom.py * geom.ld_h + (int64_t)geom.px * geom.ld_w;
-        const int64_t base = (int64_t)b * geom.ld_b + (int64_t)oys * geom.ld_h + (int64_t)oxs * geom.ld_w - shift;
-        const __amdgpu_buffer_rsrc_t rsrc = make_rsrc(geom.src + base);
-        // the padding bit of this step's case moved to bit 31: past the record count (two vector
-        // instructions per vector)
-#pragma unroll
-        for (int e = 0; e < S::kVecs; ++e)
-            buffer_into<VEC>(this->reg + e * VEC, rsrc, (((bad[e] >> flags) & 1u) << 31) | rel4[e]);
     }
 };
 
@@ -620,10 +226,10 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p) {
     using LX = std::conditional_t<
         XMODE == 0, DenseLoader<BM, BK, NT, XR, VX>,
         std::conditional_t<
-            XMODE == 1, ConvRowsLoader<BM, BK, NT, VX>,
-            std::conditional_t<XMODE == 2, ConvColsLoader<BM, BK, NT, VX>,
-                               std::conditional_t<XMODE == 3, ConvColsStepLoader<BM, BK, NT, VX>,
-                                                  ConvRowsBufferLoader<BM, BK, NT, VX>>>>>;
+            XMODE == 1, ConvRowsLoader<Staging<BM, BK, NT, true, VX>, BM, BK, NT, VX>,
+            std::conditional_t<XMODE == 2, ConvColsLoader<Staging<BM, BK, NT, false, VX>, BM, BK, NT, VX>,
+                               std::conditional_t<XMODE == 3, ConvColsStepLoader<Staging<BM, BK, NT, false, VX>, BM, BK, NT, VX>,
+                                                  ConvRowsBufferLoader<Staging<BM, BK, NT, true, VX>, BM, BK, NT, VX>>>>>;
     using LY = DenseLoader<BN, BK, NT, YR, VY>;
     constexpr int kStage = BK * LX::LD + BK * LY::LD;
     constexpr int kPoolPitch = TN + 1;
@@ -859,52 +465,7 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p) {
             }
         }
     } else if constexpr (EPI == 0) {
-        float *c = p.c + batch * p.c_batch + (int64_t)split * p.c_split;
-        // bias / axpby apply to whole sums only; split sums finish them at the end
-        const bool whole = p.splits == 1;
-        const float *bias = whole ? p.bias : nullptr;
-        const float *d = whole ? p.d : nullptr;
-        const int64_t out_base = batch * p.m * p.n;
-        const int64_t col = j0 + col_l;
-        if (p.n % FN == 0 && (reinterpret_cast<uintptr_t>(c) & (4 * FN - 1)) == 0) {
-            // one FN-wide vector store per row (col < n implies all FN columns are)
-            if (col < p.n) {
-#pragma unroll
-                for (int a = 0; a < FM; ++a)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const int64_t row = i0 + row_of(a, v);
-                        if (row >= p.m) continue;
-                        const int64_t idx = row * p.n + col;
-                        if constexpr (FN == 4) {
-                            floatx4 o;
-#pragma unroll
-                            for (int b = 0; b < 4; ++b)
-                                o[b] = finish_value(bias, d, p.alpha, p.beta, acc[a][b][v], out_base + idx + b, col + b);
-                            *reinterpret_cast<floatx4 *>(c + idx) = o;
-                        } else {
-                            float2 o;
-                            o.x = finish_value(bias, d, p.alpha, p.beta, acc[a][0][v], out_base + idx, col);
-                            o.y = finish_value(bias, d, p.alpha, p.beta, acc[a][1][v], out_base + idx + 1, col + 1);
-                            *reinterpret_cast<float2 *>(c + idx) = o;
-                        }
-                    }
-            }
-        } else {
-#pragma unroll
-            for (int b = 0; b < FN; ++b) {
-                if (col + b >= p.n) continue;
-#pragma unroll
-                for (int a = 0; a < FM; ++a)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const int64_t row = i0 + row_of(a, v);
-                        if (row < p.m)
-                            c[row * p.n + col + b] = finish_value(bias, d, p.alpha, p.beta, acc[a][b][v],
-                                                                  out_base + row * p.n + col + b, col + b);
-                    }
-            }
-        }
+        store_tile(p, acc, batch, split, i0 + wm * TM + FM * 4 * quad, j0 + col_l);
     } else {
         // The block's BM rows are whole rows of pooling windows (the host guarantees
         // BM % (pool_h * pool_ow) == 0 and an exact tiling), so every window is complete here.
@@ -913,54 +474,7 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p) {
         const int windows = BM / (kh * kw);
         const int64_t pooled_row0 = i0 / ow / kh;
         if (p.conv.window_major) {
-            // 2x2 windows, tile rows window-major: acc[a][b][v] is position a of the wave's window
-            // 4 * quad + v, so each lane pools whole windows from its own registers (no LDS, no
-            // barrier) and writes its FN adjacent columns as one vector of values and one of
-            // winner bytes.
-            float addv[FN];
-            bool okv[FN];
-#pragma unroll
-            for (int b = 0; b < FN; ++b) {
-                const int64_t col = j0 + col_l + b;
-                okv[b] = col < p.n;
-                addv[b] = (p.bias != nullptr && okv[b]) ? p.bias[col] : 0.0f;
-            }
-            const bool vec = p.n % FN == 0 && (reinterpret_cast<uintptr_t>(p.pooled) & (4 * FN - 1)) == 0 &&
-                             (reinterpret_cast<uintptr_t>(p.argmax) & (FN - 1)) == 0;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int w = wm * (TM / 4) + 4 * quad + v;  // window inside the tile
-                const int wr = (int)p.pool_cols.div((uint32_t)w), wc = w - wr * pw;
-                if (i0 + (int64_t)wr * 2 * ow >= p.m) continue;
-                float best[FN];
-                int winner[FN];
-#pragma unroll
-                for (int b = 0; b < FN; ++b) {
-                    float y[4];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) y[e] = acc[e][b][v] + addv[b];
-                    relu_pool_window4(y, best[b], winner[b]);
-                }
-                const int64_t out = ((pooled_row0 + wr) * pw + wc) * p.n + j0 + col_l;
-                if (vec && okv[0]) {
-                    if constexpr (FN == 4) {
-                        *reinterpret_cast<floatx4 *>(p.pooled + out) = floatx4{best[0], best[1], best[2], best[3]};
-                        *reinterpret_cast<uint32_t *>(p.argmax + out) =
-                            (uint32_t)winner[0] | ((uint32_t)winner[1] << 8) | ((uint32_t)winner[2] << 16) |
-                            ((uint32_t)winner[3] << 24);
-                    } else {
-                        *reinterpret_cast<float2 *>(p.pooled + out) = make_float2(best[0], best[1]);
-                        *reinterpret_cast<uint16_t *>(p.argmax + out) = (uint16_t)(winner[0] | (winner[1] << 8));
-                    }
-                } else {
-#pragma unroll
-                    for (int b = 0; b < FN; ++b) {
-                        if (!okv[b]) continue;
-                        p.pooled[out + b] = best[b];
-                        p.argmax[out + b] = (uint8_t)winner[b];
-                    }
-                }
-            }
+            pool_tile<TM>(p, acc, i0, wm, quad, j0 + col_l);
             return;
         }
         // Other windows: one column half (the waves with wn == h) at a time goes through LDS as
@@ -1218,12 +732,17 @@ enum class Shape { Large, Tall, Small, Wide };
 struct Choice {
     Shape shape;
     int bm, bn, bk, per_cu;
+    TileRate rate;
 };
+// Paces measured on 4096^3 (143 TFLOP/s), 1024^3 (64x64 tiles: 26.7 us) and the CNN's convolutions.
+constexpr Choice kLarge{Shape::Large, 128, 128, 32, 2, {2, 1.88, 2.3, 5.0}};
+constexpr Choice kTall{Shape::Tall, 128, 64, 32, 3, {3, 1.02, 1.2, 4.0}};
+constexpr Choice kSmall{Shape::Small, 64, 64, 32, 4, {4, 0.57, 0.73, 3.5}};
+constexpr Choice kWide{Shape::Wide, 64, 128, 32, 3, {3, 0.98, 1.2, 4.0}};
 
 Choice choose(int64_t m, int64_t n, int64_t k, int64_t batch, int64_t cus, bool pool_epilogue,
               bool wide_ok = false) {
-    const Choice large{Shape::Large, 128, 128, 32, 2}, tall{Shape::Tall, 128, 64, 32, 3},
-        small{Shape::Small, 64, 64, 32, 4}, wide{Shape::Wide, 64, 128, 32, 3};
+    const Choice &large = kLarge, &tall = kTall, &small = kSmall, &wide = kWide;
     if (m < 128 && !pool_epilogue) return small;
     if (n < 128) return n <= 64 || pool_epilogue ? tall : small;
     if (wide_ok) return wide;
@@ -1248,8 +767,7 @@ struct DenseSchedule {
 };
 
 DenseSchedule dense_schedule(int64_t m, int64_t n, int64_t k, int64_t batch, int64_t cus) {
-    const Choice shapes[3] = {{Shape::Large, 128, 128, 32, 2}, {Shape::Tall, 128, 64, 32, 3},
-                              {Shape::Small, 64, 64, 32, 4}};
+    const Choice shapes[3] = {kLarge, kTall, kSmall};
     const double eff[3] = {1.0, 0.96, 0.92};
     const int64_t out_len = batch * m * n;
     DenseSchedule best{shapes[0], 1};
@@ -1416,64 +934,7 @@ int run_gemm(axis_device device, GemmParams p, int64_t batch, float *out, const 
         }
     p.bf16 = device->bf16_matmul;
     const int64_t cus = device->multiprocessors;
-    Choice ch = choose(p.m, p.n, p.k, batch, cus, EPI == 1, XMODE == 3);
-    int64_t scheduled_splits = 0;
-    if constexpr (XMODE == 0 && EPI == 0) {
-        const int64_t large_tiles = ((p.m + 127) / 128) * ((p.n + 127) / 128) * batch;
-        if (!p.perm_c && large_tiles < 2 * cus && p.k >= 4 * 32) {
-            const DenseSchedule d = dense_schedule(p.m, p.n, p.k, batch, cus);
-            ch = d.choice;
-            scheduled_splits = d.splits;
-        }
-    }
-    const int BK = ch.bk;
-    p.tiles_m = static_cast<int32_t>((p.m + ch.bm - 1) / ch.bm);
-    p.tiles_n = static_cast<int32_t>((p.n + ch.bn - 1) / ch.bn);
-    const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n * batch;
-    // Split the reduction when the tiles alone cannot fill the chip (dense products: as the
-    // schedule above decided): aim at one full round of resident blocks so no round runs nearly
-    // empty.  The pooling epilogue needs whole sums.  Other reductions under 16 K steps are not
-    // split (the extra sum launch would cost more than it saves).  The partial slices stay within
-    // 64 MiB.
-    const int64_t slots = cus * ch.per_cu;
     const int64_t out_len = batch * p.m * p.n;
-    int64_t splits = 1;
-    if (scheduled_splits > 0) {
-        splits = scheduled_splits;
-    } else if (EPI == 0 && tiles < slots && p.k >= 16 * BK) {
-        splits = std::min<int64_t>({slots / tiles, p.k / (BK * 4), (int64_t(16) << 20) / out_len});
-        splits = std::max<int64_t>(splits, 1);
-    }
-    int64_t chunk = (p.k + splits - 1) / splits;
-    chunk = (chunk + BK - 1) / BK * BK;
-    if (chunk < BK) chunk = BK;
-    splits = (p.k + chunk - 1) / chunk;
-    if (splits < 1) splits = 1;
-    p.k_chunk = chunk;
-    p.splits = static_cast<int32_t>(splits);
-    // Two to four slices of at most 128 over at most one 32x32 tile per CU: one block per tile whose
-    // waves are the slices (gemm_fold_kernel), with no partial buffer and no sum launch; the same
-    // bits as the slices and their sum.  Its 64-deep stages reach 31 * s_t + 63 * s_r elements.
-    auto fold_reach = [](int64_t st, int64_t sr) { return 31 * st + 63 * sr < (int64_t(1) << 29); };
-    const int64_t fold_tiles = ((p.m + 31) / 32) * ((p.n + 31) / 32) * batch;
-    const bool fold = XMODE == 0 && EPI == 0 && scheduled_splits > 1 && ch.shape == Shape::Small && splits >= 2 &&
-                      splits <= 4 && chunk <= 128 && fold_tiles <= cus && !p.perm_c && device->fold_splits &&
-                      fold_reach(p.x_si, p.x_sr) && fold_reach(p.y_sj, p.y_sr);
-    if (fold) {
-        p.tiles_m = static_cast<int32_t>((p.m + 31) / 32);
-        p.tiles_n = static_cast<int32_t>((p.n + 31) / 32);
-    }
-
-    // Dense operands read through 32-bit offsets inside a tile: at most 127 * s_t + 31 * s_r elements.
-    auto reach = [](int64_t st, int64_t sr) { return st >= 0 && sr >= 0 && 127 * st + 31 * sr < (int64_t(1) << 29); };
-    if (XMODE == 0 && !reach(p.x_si, p.x_sr))
-        return axis::fail(AXIS_ERROR_INVALID, "matmul operand row pitch must stay below 4,227,000 elements");
-    if (!reach(p.y_sj, p.y_sr))
-        return axis::fail(AXIS_ERROR_INVALID, "matmul operand row pitch must stay below 4,227,000 elements");
-    // t-contiguous dense operands bound a K step's rows by the resource's record count: unit
-    // element stride and rows no longer than their pitch (every entry point lays them out so)
-    if ((XMODE == 0 && !XR && (p.x_si != 1 || p.x_sr < p.m)) || (!YR && (p.y_sj != 1 || p.y_sr < p.n)))
-        return axis::fail(AXIS_ERROR_INVALID, "t-contiguous product operand without unit stride and full-row pitch");
     bool vx;
     if constexpr (XMODE == 0)
         vx = XR ? vec_ok(p.x, p.k, p.x_si) && p.x_batch % 4 == 0
@@ -1483,6 +944,90 @@ int run_gemm(axis_device device, GemmParams p, int64_t batch, float *out, const 
              p.conv.ld_w % 4 == 0 && p.conv.ld_h % 4 == 0 && p.conv.ld_b % 4 == 0;
     const bool vy = YR ? vec_ok(p.y, p.k, p.y_sj) && p.y_batch % 4 == 0
                        : vec_ok(p.y, p.n, p.y_sr) && p.y_batch % 4 == 0;
+    // Dense operands are read through 32-bit offsets inside a tile: at most (rows - 1) * s_t + 31 * s_r elements.
+    auto reach = [](int64_t rows, int64_t st, int64_t sr) {
+        return st >= 0 && sr >= 0 && (rows - 1) * st + 31 * sr < (int64_t(1) << 29);
+    };
+    Choice ch = choose(p.m, p.n, p.k, batch, cus, EPI == 1, XMODE == 3);
+    int64_t splits = 1;
+    bool scheduled = false;
+    if constexpr (XMODE == 0 && EPI == 0) {
+        const int64_t large_tiles = ((p.m + 127) / 128) * ((p.n + 127) / 128) * batch;
+        if (!p.perm_c && large_tiles < 2 * cus && p.k >= 4 * 32) {
+            const DenseSchedule d = dense_schedule(p.m, p.n, p.k, batch, cus);
+            ch = d.choice;
+            splits = d.splits;
+            scheduled = true;
+        }
+    }
+    const int BK = ch.bk;
+    int64_t tiles = ((p.m + ch.bm - 1) / ch.bm) * ((p.n + ch.bn - 1) / ch.bn) * batch;
+    // Split the reduction when the tiles alone cannot fill the chip (dense products: as the
+    // schedule above decided): aim at one full round of resident blocks so no round runs nearly
+    // empty.  The pooling epilogue needs whole sums.  Other reductions under 16 K steps are not
+    // split (the extra sum launch would cost more than it saves).  The partial slices stay within
+    // 64 MiB.
+    const int64_t slots = cus * ch.per_cu;
+    if (!scheduled && EPI == 0 && tiles < slots && p.k >= 16 * BK) {
+        splits = std::min<int64_t>({slots / tiles, p.k / (BK * 4), (int64_t(16) << 20) / out_len});
+        splits = std::max<int64_t>(splits, 1);
+    }
+    auto cut = [&]() {
+        int64_t chunk = (p.k + splits - 1) / splits;
+        chunk = (chunk + BK - 1) / BK * BK;
+        if (chunk < BK) chunk = BK;
+        splits = (p.k + chunk - 1) / chunk;
+        if (splits < 1) splits = 1;
+        p.k_chunk = chunk;
+        p.splits = static_cast<int32_t>(splits);
+    };
+    cut();
+    // Two to four slices of at most 128 over at most one 32x32 tile per CU: one block per tile whose
+    // waves are the slices (gemm_fold_kernel), with no partial buffer and no sum launch; the same
+    // bits as the slices and their sum.  Its 64-deep stages reach 31 * s_t + 63 * s_r elements.
+    auto fold_reach = [](int64_t st, int64_t sr) { return 31 * st + 63 * sr < (int64_t(1) << 29); };
+    const int64_t fold_tiles = ((p.m + 31) / 32) * ((p.n + 31) / 32) * batch;
+    const bool foldable = XMODE == 0 && EPI == 0 && scheduled && ch.shape == Shape::Small && splits >= 2 &&
+                          splits <= 4 && p.k_chunk <= 128 && fold_tiles <= cus && !p.perm_c &&
+                          fold_reach(p.x_si, p.x_sr) && fold_reach(p.y_sj, p.y_sr);
+    const bool fold = foldable && device->fold_splits;
+    // The larger launches of an fp32 handle take the bf16 matrix cores on split operands
+    // (gemm_split.hip), where their estimate is below this kernel's; convolutions need vector loads
+    // there.  Foldable products are latency on either.  The fused forward stays here: its winners are
+    // whole numbers, and another rounding of the sums moves those of windows that tie to rounding.
+    // Forward convolutions of fewer than 256 terms stay too: there the plain and the fused entry agree
+    // bit for bit.
+    SplitPlan planes;
+    const int xmode = XMODE == 4 && !p.conv.tap_steps ? 5 : XMODE;  // gemm_split.hip's rows modes
+    if (XMODE != 1 && EPI == 0 && !p.bf16 && !foldable && (XMODE == 0 || (vx && vy)) &&
+        !(XMODE == 4 && !YR && p.k < 256) && (XMODE != 0 || reach(256, p.x_si, p.x_sr)) &&
+        reach(256, p.y_sj, p.y_sr)) {
+        // (single-element loads run about 15% slower; 3%: leave a tie here)
+        const double us = launch_us(tiles * splits, (double)(p.k_chunk / BK), ch.rate, cus) *
+                              ((XMODE != 0 || vx) && vy ? 1.0 : 1.15) +
+                          slices_us(splits, out_len);
+        planes = split_plan(p.m, p.n, p.k, batch, cus, YR, vx && vy, xmode, 0.97 * us);
+    }
+    const bool on_planes = planes.tile != SplitTile::None;
+    if (on_planes) {
+        ch.bm = planes.rows;
+        ch.bn = planes.cols;
+        splits = planes.splits;
+        cut();
+    }
+    p.tiles_m = static_cast<int32_t>((p.m + ch.bm - 1) / ch.bm);
+    p.tiles_n = static_cast<int32_t>((p.n + ch.bn - 1) / ch.bn);
+    if (fold) {
+        p.tiles_m = static_cast<int32_t>((p.m + 31) / 32);
+        p.tiles_n = static_cast<int32_t>((p.n + 31) / 32);
+    }
+
+    if ((XMODE == 0 && !reach(128, p.x_si, p.x_sr)) || !reach(128, p.y_sj, p.y_sr))
+        return axis::fail(AXIS_ERROR_INVALID, "matmul operand row pitch must stay below 4,227,000 elements");
+    // t-contiguous dense operands bound a K step's rows by the resource's record count: unit
+    // element stride and rows no longer than their pitch (every entry point lays them out so)
+    if ((XMODE == 0 && !XR && (p.x_si != 1 || p.x_sr < p.m)) || (!YR && (p.y_sj != 1 || p.y_sr < p.n)))
+        return axis::fail(AXIS_ERROR_INVALID, "t-contiguous product operand without unit stride and full-row pitch");
 
     axis::Scratch partial, ordered;
     // spare: the range sums of more than 32 slices, or an unsplit permuted product before its move
@@ -1527,7 +1072,11 @@ int run_gemm(axis_device device, GemmParams p, int64_t batch, float *out, const 
     const double k_work = (double)(p.k_work > 0 ? p.k_work : p.k);
     axis::TimedLaunch timed(ws ? nullptr : device, "gemm", 2.0 * (double)batch * (double)p.m * (double)p.n * k_work);
     dim3 grid(static_cast<unsigned>(blocks));
-    if (fold) {
+    int status = AXIS_OK;
+    if (on_planes) {
+        if (xmode == 4 && !p.ytaps.on) p.ytaps = TapSteps::rows(p.y_sr);
+        status = split_gemm(device, p, planes.tile, XR, YR, vx && vy, xmode, grid.x);
+    } else if (fold) {
         if constexpr (XMODE == 0 && EPI == 0) launch_fold<XR, YR>(p, grid, device->stream, vx, vy);
     } else if constexpr (EPI == 1) {
         // the fused forward's 128x128 tiles in eight waves of 64x32 (307.8 -> 302.8 us per launch)
@@ -1554,7 +1103,7 @@ int run_gemm(axis_device device, GemmParams p, int64_t batch, float *out, const 
         else if constexpr (XMODE == 3)  // Wide: cols-mode weight gradients only
             launch_vec<64, 128, 32, 2, 2, XR, YR, XMODE, EPI>(p, grid, device->stream, vx, vy);
     }
-    int status = axis::launch_status("gemm_kernel");
+    if (!on_planes) status = axis::launch_status("gemm_kernel");
     if (status) return status;
     if (splits > 1 && !fold)
         status = sum_splits(device, partials, out, out_len, splits, p.bias, p.n, p.d, p.alpha, p.beta,
@@ -1710,8 +1259,7 @@ int forward_weight(axis_device device, const float *weight, const ConvShape &s, 
         p.y = weight;
         p.y_sj = 1;
         p.y_sr = taps * s.out_channels;
-        p.ytaps = TapSteps{true, FastDiv((uint32_t)s.channels), taps * s.out_channels, s.out_channels, 0, block,
-                           FastDiv((uint32_t)taps)};
+        p.ytaps = TapSteps::make(block, s.channels, taps, taps * s.out_channels, s.out_channels, 0);
         return AXIS_OK;
     }
     if (int st = permuted.get(device, sizeof(float) * (size_t)(c_pad * taps * s.out_channels))) return st;
@@ -2055,8 +1603,7 @@ int axis_conv2d_backward_data(axis_device device, const float *gradient, const f
         p.y = weight;
         p.y_sr = 1;
         p.y_sj = taps * out_channels;
-        p.ytaps = TapSteps{true, FastDiv((uint32_t)out_channels), 1, -(int64_t)out_channels,
-                           (taps - 1) * out_channels, block, FastDiv((uint32_t)taps)};
+        p.ytaps = TapSteps::make(block, out_channels, taps, 1, -(int64_t)out_channels, (taps - 1) * out_channels);
         return buffered ? run_gemm<true, true, 4, 0>(device, p, 1, d_input)
                         : run_gemm<true, true, 1, 0>(device, p, 1, d_input);
     }
