@@ -8,6 +8,23 @@
 
 namespace axis {
 
+// Sum in row order of a column staged in LDS, rows PITCH floats apart (a multiple of 32 of them, the
+// ones past n_rows zero: adding them changes no bit, the sum is never -0).  32 rows are read before
+// they are added: one LDS latency per 32 dependent adds instead of one per add.
+template <int PITCH>
+__device__ __forceinline__ float staged_column_sum(const float *column, int n_rows) {
+    constexpr int kAhead = 32;
+    float sum = 0.0f;
+    for (int r = 0; r < n_rows; r += kAhead) {
+        float v[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) v[u] = column[(r + u) * PITCH];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) sum = sum + v[u];
+    }
+    return sum;
+}
+
 typedef float floatx4_cs __attribute__((ext_vector_type(4)));
 constexpr int kCombineStage = 4096;
 

@@ -396,49 +396,57 @@ struct BiasAdd {
 
 // Stage one of the bias gradient: partial[q][c] = sum of rows [512q, 512q+512) of column c,
 // sequentially; optionally masked by relu_input > 0 (and the masked gradient written out).
-// Block (column group, chunk): the chunk's rows of 16 columns are staged in LDS first -- every
-// load of the chunk in flight at once, coalesced in 64-byte row segments -- then one lane per
-// column adds its 512 (or fewer) rows in row order.  A lane summing straight from memory waits on
-// one round trip per batch of loads: 8.4 us for a [256, 1000] gradient against ~3 us staged.
-constexpr int kChunkCols = 8;
-template <bool MASK>
+// Block (COLS columns, chunk): the chunk's rows are staged in LDS first -- every load of the chunk in
+// flight at once, in row segments of 4 COLS bytes -- then one lane per column adds its rows in row
+// order (staged_column_sum).  32 columns make whole 128-byte lines; 8 give small operands more
+// blocks.  Bound by HBM and the 512 dependent adds (about 2 us); measured with the combine, against
+// sums that read LDS one row at a time: [8192, 1024] 28 -> 10 us, [1531, 2049] 28 -> 10 us,
+// [4096, 4096] 30 -> 21 us, masked [8192, 1024] 60 -> 33 us.
+constexpr int kChunkCols = 8, kChunkColsWide = 32;
+template <int COLS, bool MASK>
 __global__ void __launch_bounds__(kBlock) column_chunk_kernel(const float *__restrict__ g,
                                                               const float *__restrict__ relu_input,
                                                               float *__restrict__ masked_out,
                                                               float *__restrict__ partial,
                                                               int64_t rows, int64_t width, int64_t chunks,
                                                               float *__restrict__ out) {
-    static_assert(axis::kGroupedChunk * kChunkCols % kBlock == 0, "whole staging passes");
-    constexpr int kPasses = axis::kGroupedChunk * kChunkCols / kBlock;
-    constexpr int kRowsPerPass = kBlock / kChunkCols;
-    __shared__ float staged[axis::kGroupedChunk][kChunkCols + 1];
+    static_assert(axis::kGroupedChunk * COLS % kBlock == 0, "whole staging passes");
+    constexpr int kPasses = axis::kGroupedChunk * COLS / kBlock;
+    constexpr int kRowsPerPass = kBlock / COLS;
+    __shared__ float staged[axis::kGroupedChunk * (COLS + 1)];
     const int tid = threadIdx.x;
-    const int cl = tid % kChunkCols;
-    const int64_t c = (int64_t)blockIdx.x * kChunkCols + cl;
+    const int cl = tid % COLS;
+    const int64_t c = (int64_t)blockIdx.x * COLS + cl;
     for (int64_t q = blockIdx.y; q < chunks; q += gridDim.y) {
         const int64_t r0 = q * axis::kGroupedChunk;
         const int n_rows = (int)(r0 + axis::kGroupedChunk < rows ? axis::kGroupedChunk : rows - r0);
-        float v[kPasses];
-#pragma unroll
-        for (int u = 0; u < kPasses; ++u) {
-            const int r = u * kRowsPerPass + tid / kChunkCols;
-            v[u] = 0.0f;
-            if (r < n_rows && c < width) {
-                const int64_t idx = (r0 + r) * width + c;
-                v[u] = g[idx];
-                if (MASK) {
-                    v[u] = relu_input[idx] > 0.0f ? v[u] : 0.0f;
-                    masked_out[idx] = v[u];
-                }
-            }
-        }
         __syncthreads();  // the previous chunk's sums have read the stage
+        // Passes in groups, every load of a group before its first store (loads and stores share one
+        // counter: a wait between them would serialise the passes); a masked group holds two operands.
+        constexpr int kGroup = MASK && kPasses > 16 ? 16 : kPasses;
+#pragma unroll 1
+        for (int u0 = 0; u0 < kPasses; u0 += kGroup) {
+            float v[kGroup], x[MASK ? kGroup : 1];
+            auto row = [&](int u) { return (u0 + u) * kRowsPerPass + tid / COLS; };
+            auto live = [&](int u) { return row(u) < n_rows && c < width; };
 #pragma unroll
-        for (int u = 0; u < kPasses; ++u) staged[u * kRowsPerPass + tid / kChunkCols][cl] = v[u];
+            for (int u = 0; u < kGroup; ++u) {
+                const int64_t idx = (r0 + row(u)) * width + c;
+                v[u] = live(u) ? g[idx] : 0.0f;
+                if (MASK) x[u] = live(u) ? relu_input[idx] : 0.0f;
+            }
+            if (MASK)
+#pragma unroll
+                for (int u = 0; u < kGroup; ++u) {
+                    v[u] = x[u] > 0.0f ? v[u] : 0.0f;
+                    if (live(u)) masked_out[(r0 + row(u)) * width + c] = v[u];
+                }
+#pragma unroll
+            for (int u = 0; u < kGroup; ++u) staged[row(u) * (COLS + 1) + cl] = v[u];
+        }
         __syncthreads();
-        if (tid < kChunkCols && c < width) {
-            float sum = 0.0f;
-            for (int r = 0; r < n_rows; ++r) sum = sum + staged[r][tid];
+        if (tid < COLS && c < width) {
+            const float sum = axis::staged_column_sum<COLS + 1>(staged + tid, n_rows);
             // A single chunk is also the whole sum: the combine's 0 + p0 (scale 1) written here.
             if (out)
                 out[c] = 0.0f + sum;
@@ -448,28 +456,27 @@ __global__ void __launch_bounds__(kBlock) column_chunk_kernel(const float *__res
     }
 }
 
-// The same chunk sums for wide operands: 64 columns per block, so every row read (and masked
-// write) is one 256-byte segment per wave.  A chunk's 512 rows pass through LDS 128 at a time;
-// wave 0's lane per column keeps adding in row order across the passes, so each sum has the
-// association of column_chunk_kernel.
-constexpr int kWideCols = 64, kWideRows = 128;
-template <bool MASK>
-__global__ void __launch_bounds__(kBlock) column_chunk_wide_kernel(const float *__restrict__ g,
-                                                                   const float *__restrict__ relu_input,
-                                                                   float *__restrict__ masked_out,
-                                                                   float *__restrict__ partial, int64_t rows,
-                                                                   int64_t width, int64_t chunks,
-                                                                   float *__restrict__ out) {
-    static_assert(kBlock == 256 && kWideRows % 4 == 0, "four waves stage whole row groups");
-    constexpr int kPerLane = kWideRows / 4;
-    __shared__ float staged[kWideRows][kWideCols + 1];
+// The masked sums of operands whose three streams pass the 256 MB last-level cache: 64 columns per
+// block, so that every row segment of the two reads and the write is 256 bytes, a chunk's rows through
+// LDS 128 at a time; wave 0's lane per column keeps adding in row order across the passes.
+// [4096, 8192]: 120 us against 175 in column_chunk_kernel; [4096, 4096]: 64 against 57.
+constexpr int kMaskCols = 64, kMaskRows = 128;
+__global__ void __launch_bounds__(kBlock) column_chunk_masked_kernel(const float *__restrict__ g,
+                                                                     const float *__restrict__ relu_input,
+                                                                     float *__restrict__ masked_out,
+                                                                     float *__restrict__ partial, int64_t rows,
+                                                                     int64_t width, int64_t chunks,
+                                                                     float *__restrict__ out) {
+    static_assert(kBlock == 256 && kMaskRows % 4 == 0, "four waves stage whole row groups");
+    constexpr int kPerLane = kMaskRows / 4;
+    __shared__ float staged[kMaskRows * (kMaskCols + 1)];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t c = (int64_t)blockIdx.x * kWideCols + lane;
+    const int64_t c = (int64_t)blockIdx.x * kMaskCols + lane;
     for (int64_t q = blockIdx.y; q < chunks; q += gridDim.y) {
         const int64_t r0 = q * axis::kGroupedChunk;
         const int n_rows = (int)(r0 + axis::kGroupedChunk < rows ? axis::kGroupedChunk : rows - r0);
         float sum = 0.0f;
-        for (int base = 0; base < n_rows; base += kWideRows) {
+        for (int base = 0; base < n_rows; base += kMaskRows) {
             float v[kPerLane];
 #pragma unroll
             for (int u = 0; u < kPerLane; ++u) {
@@ -478,19 +485,17 @@ __global__ void __launch_bounds__(kBlock) column_chunk_wide_kernel(const float *
                 if (r < n_rows && c < width) {
                     const int64_t idx = (r0 + r) * width + c;
                     v[u] = g[idx];
-                    if (MASK) {
-                        v[u] = relu_input[idx] > 0.0f ? v[u] : 0.0f;
-                        masked_out[idx] = v[u];
-                    }
+                    v[u] = relu_input[idx] > 0.0f ? v[u] : 0.0f;
+                    masked_out[idx] = v[u];
                 }
             }
             __syncthreads();  // the previous pass's sums have read the stage
 #pragma unroll
-            for (int u = 0; u < kPerLane; ++u) staged[4 * u + wave][lane] = v[u];
+            for (int u = 0; u < kPerLane; ++u) staged[(4 * u + wave) * (kMaskCols + 1) + lane] = v[u];
             __syncthreads();
             if (wave == 0 && c < width) {
-                const int lim = n_rows - base < kWideRows ? n_rows - base : kWideRows;
-                for (int r = 0; r < lim; ++r) sum = sum + staged[r][lane];
+                const int lim = n_rows - base < kMaskRows ? n_rows - base : kMaskRows;
+                for (int r = 0; r < lim; ++r) sum = sum + staged[r * (kMaskCols + 1) + lane];
             }
         }
         if (wave == 0 && c < width) {
@@ -870,25 +875,23 @@ int axis_bias_gradient(axis_device device, const float *gradient, const float *r
     if (chunks > 1)
         if (int s = partial.get(device, sizeof(float) * (size_t)pairs)) return s;
     float *direct = chunks == 1 ? out : nullptr;
-    if (width >= 2048) {  // enough 64-column blocks to fill the chip
-        const dim3 grid((unsigned)((width + kWideCols - 1) / kWideCols), (unsigned)std::min<int64_t>(chunks, 65535));
-        if (relu_input)
-            column_chunk_wide_kernel<true><<<grid, kBlock, 0, device->stream>>>(
-                gradient, relu_input, masked_out, partial.as<float>(), rows, width, chunks, direct);
-        else
-            column_chunk_wide_kernel<false><<<grid, kBlock, 0, device->stream>>>(
-                gradient, nullptr, nullptr, partial.as<float>(), rows, width, chunks, direct);
-        if (int s = axis::launch_status("column_chunk_wide_kernel")) return s;
-    } else {
-        const dim3 grid((unsigned)((width + kChunkCols - 1) / kChunkCols), (unsigned)std::min<int64_t>(chunks, 65535));
-        if (relu_input)
-            column_chunk_kernel<true><<<grid, kBlock, 0, device->stream>>>(
-                gradient, relu_input, masked_out, partial.as<float>(), rows, width, chunks, direct);
-        else
-            column_chunk_kernel<false><<<grid, kBlock, 0, device->stream>>>(
-                gradient, nullptr, nullptr, partial.as<float>(), rows, width, chunks, direct);
-        if (int s = axis::launch_status("column_chunk_kernel")) return s;
-    }
+    // whole lines where that leaves a block for every other CU
+    const bool wide = ((width + kChunkColsWide - 1) / kChunkColsWide) * chunks * 2 >= device->multiprocessors;
+    const int cols = wide ? kChunkColsWide : kChunkCols;
+    const dim3 grid((unsigned)((width + cols - 1) / cols), (unsigned)std::min<int64_t>(chunks, 65535));
+    auto launch = [&](auto kernel) {
+        kernel<<<grid, kBlock, 0, device->stream>>>(gradient, relu_input, masked_out, partial.as<float>(), rows, width,
+                                                    chunks, direct);
+    };
+    if (relu_input && 12 * rows * width > (int64_t(256) << 20)) {
+        const dim3 masked((unsigned)((width + kMaskCols - 1) / kMaskCols), (unsigned)std::min<int64_t>(chunks, 65535));
+        column_chunk_masked_kernel<<<masked, kBlock, 0, device->stream>>>(gradient, relu_input, masked_out,
+                                                                        partial.as<float>(), rows, width, chunks, direct);
+    } else if (wide)
+        relu_input ? launch(column_chunk_kernel<kChunkColsWide, true>) : launch(column_chunk_kernel<kChunkColsWide, false>);
+    else
+        relu_input ? launch(column_chunk_kernel<kChunkCols, true>) : launch(column_chunk_kernel<kChunkCols, false>);
+    if (int s = axis::launch_status("column_chunk_kernel")) return s;
     if (chunks == 1) return AXIS_OK;
     axis::column_combine_kernel<<<(unsigned)width, 256, 0, device->stream>>>(partial.as<float>(), chunks,
                                                                            width, 1.0f, out);

@@ -154,44 +154,49 @@ __global__ void __launch_bounds__(kBlock) ce_backward_kernel(const float *__rest
         out[p] = (mean_factor != 0.0f ? g_all : gradient[p / width]) * (probability[p] - targets[p]);
 }
 
-// The mean cross-entropy backward with the bias gradient of the logits' producer: block (16
+// The mean cross-entropy backward with the bias gradient of the logits' producer: block (COLS
 // columns, 512-row chunk) computes its chunk's gradient values (as ce_backward_kernel), writes them
 // and stages them in LDS; one lane per column then adds the chunk's rows in row order -- the
-// column sums of axis_bias_gradient (chunk partials combined in chunk order when rows > 512).
-constexpr int kBiasCols = 8;
+// column sums of axis_bias_gradient (chunk partials combined in chunk order when rows > 512).  Bound
+// by latency at small sizes (LDS reads 32 ahead of the adds, [256, 1000]: 5.9 -> 4.9 us) and by HBM at
+// large ones (whole lines, loads before stores, [4096, 4096]: 110 -> 53 us).
+constexpr int kBiasCols = 8, kBiasColsWide = 32;
 constexpr int kBiasChunk = axis::kGroupedChunk;
+template <int COLS>
 __global__ void __launch_bounds__(kBlock) ce_backward_mean_bias_kernel(
     const float *__restrict__ gradient, float mean_factor, const float *__restrict__ probability,
     const float *__restrict__ targets, float *__restrict__ out, float *__restrict__ partial,
     float *__restrict__ d_bias, int64_t rows, int64_t width, int64_t chunks) {
-    constexpr int kPasses = kBiasChunk * kBiasCols / kBlock;
-    constexpr int kRowsPerPass = kBlock / kBiasCols;
-    __shared__ float staged[kBiasChunk][kBiasCols + 1];
+    constexpr int kPasses = kBiasChunk * COLS / kBlock;
+    constexpr int kRowsPerPass = kBlock / COLS;
+    __shared__ float staged[kBiasChunk * (COLS + 1)];
     const int tid = threadIdx.x;
-    const int cl = tid % kBiasCols;
-    const int64_t c = (int64_t)blockIdx.x * kBiasCols + cl;
+    const int cl = tid % COLS;
+    const int64_t c = (int64_t)blockIdx.x * COLS + cl;
     const float g = gradient[0] * mean_factor;
     for (int64_t q = blockIdx.y; q < chunks; q += gridDim.y) {
         const int64_t r0 = q * kBiasChunk;
         const int n_rows = (int)(r0 + kBiasChunk < rows ? kBiasChunk : rows - r0);
-        float v[kPasses];
+        float v[kPasses], t[kPasses];
+        auto row = [&](int u) { return u * kRowsPerPass + tid / COLS; };
+        auto live = [&](int u) { return row(u) < n_rows && c < width; };
 #pragma unroll
         for (int u = 0; u < kPasses; ++u) {
-            const int r = u * kRowsPerPass + tid / kBiasCols;
-            v[u] = 0.0f;
-            if (r < n_rows && c < width) {
-                const int64_t p = (r0 + r) * width + c;
-                v[u] = g * (probability[p] - targets[p]);
-                out[p] = v[u];
-            }
+            const int64_t p = (r0 + row(u)) * width + c;
+            v[u] = live(u) ? probability[p] : 0.0f;
+            t[u] = live(u) ? targets[p] : 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < kPasses; ++u) {
+            v[u] = live(u) ? g * (v[u] - t[u]) : 0.0f;
+            if (live(u)) out[(r0 + row(u)) * width + c] = v[u];
         }
         __syncthreads();  // the previous chunk's sums have read the stage
 #pragma unroll
-        for (int u = 0; u < kPasses; ++u) staged[u * kRowsPerPass + tid / kBiasCols][cl] = v[u];
+        for (int u = 0; u < kPasses; ++u) staged[row(u) * (COLS + 1) + cl] = v[u];
         __syncthreads();
-        if (tid < kBiasCols && c < width) {
-            float sum = 0.0f;
-            for (int r = 0; r < n_rows; ++r) sum = sum + staged[r][tid];
+        if (tid < COLS && c < width) {
+            const float sum = axis::staged_column_sum<COLS + 1>(staged + tid, n_rows);
             if (chunks == 1)
                 d_bias[c] = 0.0f + sum;
             else
@@ -267,10 +272,15 @@ int axis_categorical_cross_entropy_backward_mean(axis_device device, const float
     axis::Scratch partial;
     if (chunks > 1)
         if (int s = partial.get(device, sizeof(float) * (size_t)(chunks * width))) return s;
-    const dim3 grid((unsigned)((width + kBiasCols - 1) / kBiasCols), (unsigned)std::min<int64_t>(chunks, 65535));
-    ce_backward_mean_bias_kernel<<<grid, kBlock, 0, device->stream>>>(gradient, factor, probability, targets, out,
-                                                                    partial.as<float>(), d_bias, rows, width,
-                                                                    chunks);
+    // 32 columns (whole 128-byte lines) where that leaves a block for every other CU
+    const bool wide = ((width + kBiasColsWide - 1) / kBiasColsWide) * chunks * 2 >= device->multiprocessors;
+    const int cols = wide ? kBiasColsWide : kBiasCols;
+    const dim3 grid((unsigned)((width + cols - 1) / cols), (unsigned)std::min<int64_t>(chunks, 65535));
+    auto launch = [&](auto kernel) {
+        kernel<<<grid, kBlock, 0, device->stream>>>(gradient, factor, probability, targets, out, partial.as<float>(),
+                                                    d_bias, rows, width, chunks);
+    };
+    wide ? launch(ce_backward_mean_bias_kernel<kBiasColsWide>) : launch(ce_backward_mean_bias_kernel<kBiasCols>);
     if (int s = axis::launch_status("ce_backward_mean_bias_kernel")) return s;
     if (chunks == 1) return AXIS_OK;
     axis::column_combine_kernel<<<(unsigned)width, 256, 0, device->stream>>>(partial.as<float>(), chunks, width,

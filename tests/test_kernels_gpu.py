@@ -481,8 +481,8 @@ def test_adam_multi_many_tensors(dev, oracle):
 
 # ---------------------------------------------------------------- fused entries
 
-# the last three take the 64-column kernel (widths from 2048): ragged columns over three chunks,
-# one chunk written directly, config 5's [4096, 8192] layer
+# the last three are wide: ragged columns over three chunks, one chunk written directly, config 5's
+# [4096, 8192] layer (masked sums past the last-level cache)
 @pytest.mark.parametrize("rows,width", [(1, 1), (600, 2), (1030, 64), (777, 130), (1300, 2100), (300, 4096),
                                         (4096, 8192)])
 def test_bias_entries_bit_exact(dev, oracle, rows, width):
