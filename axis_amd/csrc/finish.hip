@@ -42,7 +42,7 @@ __global__ void __launch_bounds__(256) finish_batch_kernel(FinishBatch b) {
         acc[group][lane] = axis::split_sum_part4(k.partial, i4, k.len, (int32_t)k.count, k.stride, group);
         __syncthreads();
         if (group == 0 && i4 < k.len) {
-            axis::split_sum_store4(k.out_a, i4, acc[0][lane], acc[1][lane], acc[2][lane], acc[3][lane], k.bias, k.n,
+            axis::split_sum_store4(k.out_a, i4, k.len, acc[0][lane], acc[1][lane], acc[2][lane], acc[3][lane], k.bias, k.n,
                                    k.d, k.alpha, k.beta, k.perm_c, k.perm_taps);
         }
     } else if (k.kind == 0) {

@@ -68,8 +68,9 @@ __device__ __forceinline__ float split_sum_part(const float *__restrict__ partia
 
 typedef float finish_floatx4 __attribute__((ext_vector_type(4)));
 
-// The same sums for four consecutive outputs i4 .. i4 + 3 per lane (len % 4 == 0 and 16-byte
-// aligned slices): one 16-byte load per slice, each output's adds in the same order.
+// The same sums for four consecutive outputs i4 .. i4 + 3 per lane (16-byte aligned slices a multiple of
+// four floats apart, so that the last vector ends inside its slice): one 16-byte load per slice, each
+// output's adds in the same order.
 __device__ __forceinline__ finish_floatx4 split_sum_part4(const float *__restrict__ partial, int64_t i4, int64_t len,
                                                           int32_t splits, int64_t split_stride, int group) {
     constexpr int kAhead = 8;
@@ -102,17 +103,19 @@ __device__ __forceinline__ void split_sum_store(float *__restrict__ out, int64_t
     out[at] = finish_value(bias, d, alpha, beta, total, i, i % n);
 }
 
-// split_sum_store for outputs i4 .. i4 + 3 (group sums g0..g3 per output): one 16-byte store when
-// the outputs are not permuted.
-__device__ __forceinline__ void split_sum_store4(float *__restrict__ out, int64_t i4, finish_floatx4 g0,
+// split_sum_store for outputs i4 .. i4 + 3 below len (group sums g0..g3 per output): one 16-byte store
+// when the outputs are not permuted and all four are there.
+__device__ __forceinline__ void split_sum_store4(float *__restrict__ out, int64_t i4, int64_t len, finish_floatx4 g0,
                                                  finish_floatx4 g1, finish_floatx4 g2, finish_floatx4 g3,
                                                  const float *__restrict__ bias, int64_t n,
                                                  const float *__restrict__ d, float alpha, float beta,
                                                  int32_t perm_c, int32_t perm_taps) {
-    if (perm_c) {
+    if (perm_c || i4 + 4 > len) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-            split_sum_store(out, i4 + e, g0[e], g1[e], g2[e], g3[e], bias, n, d, alpha, beta, perm_c, perm_taps);
+            if (i4 + e < len)
+                split_sum_store(out, i4 + e, g0[e], g1[e], g2[e], g3[e], bias, n, d, alpha, beta, perm_c,
+                                perm_taps);
         return;
     }
     finish_floatx4 v;

@@ -561,8 +561,8 @@ __global__ void __launch_bounds__(256) split_sum_kernel(const float *__restrict_
                               beta, perm_c, perm_taps);
 }
 
-// split_sum_kernel for len % 4 == 0 over 16-byte aligned slices: 256 outputs per block, four per
-// lane, the same association per output.
+// split_sum_kernel over 16-byte aligned slices a multiple of four floats apart: 256 outputs per block,
+// four per lane, the same association per output ([1531, 1023] in five slices: 16 -> 8 us).
 __global__ void __launch_bounds__(256) split_sum4_kernel(const float *__restrict__ partial,
                                                          float *__restrict__ out, int64_t len,
                                                          int32_t splits, int64_t split_stride,
@@ -575,14 +575,14 @@ __global__ void __launch_bounds__(256) split_sum4_kernel(const float *__restrict
     acc[group][lane] = axis::split_sum_part4(partial, i4, len, splits, split_stride, group);
     __syncthreads();
     if (group == 0 && i4 < len) {
-        axis::split_sum_store4(out, i4, acc[0][lane], acc[1][lane], acc[2][lane], acc[3][lane], bias, n, d, alpha,
+        axis::split_sum_store4(out, i4, len, acc[0][lane], acc[1][lane], acc[2][lane], acc[3][lane], bias, n, d, alpha,
                                beta, perm_c, perm_taps);
     }
 }
 
-// First level for many slices: mid[g][i] = sum of slices [g*span, (g+1)*span) in order.
+// First level for many slices (and their sums) `stride` apart: mid[g][i] = sum of slices [g*span, (g+1)*span) in order.
 __global__ void __launch_bounds__(256) split_range_kernel(const float *__restrict__ partial,
-                                                          float *__restrict__ mid, int64_t len,
+                                                          float *__restrict__ mid, int64_t len, int64_t stride,
                                                           int32_t splits, int32_t span) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= len) return;
@@ -594,12 +594,12 @@ __global__ void __launch_bounds__(256) split_range_kernel(const float *__restric
     for (int32_t k0 = g * span; k0 < k1; k0 += kAhead) {
         float v[kAhead];
 #pragma unroll
-        for (int u = 0; u < kAhead; ++u) v[u] = k0 + u < k1 ? partial[(int64_t)(k0 + u) * len + i] : 0.f;
+        for (int u = 0; u < kAhead; ++u) v[u] = k0 + u < k1 ? partial[(int64_t)(k0 + u) * stride + i] : 0.f;
 #pragma unroll
         for (int u = 0; u < kAhead; ++u)
             if (k0 + u < k1) s += v[u];
     }
-    mid[(int64_t)g * len + i] = s;
+    mid[(int64_t)g * stride + i] = s;
 }
 
 // Weight permutations between the reference's [(c, ky, kx), n] layout and the implicit-GEMM
@@ -801,18 +801,22 @@ DenseSchedule dense_schedule(int64_t m, int64_t n, int64_t k, int64_t batch, int
     return best;
 }
 
+// Slices start on 16 bytes: up to three floats between the end of one and the next.
+int64_t slice_stride(int64_t len) { return (len + 3) / 4 * 4; }
+
 // Deterministic sum of reduction slices (+ bias): up to 32 slices in one pass; beyond that, ranges
 // of 32 consecutive slices first, then the range sums -- a fixed association for a given count.
+// stride: floats between slices (slice_stride).
 // `owner` (the block holding `partial`), when given and the handle defers finishing sums, lets
 // the last pass be recorded instead of launched: `out` is then a final gradient.
-int sum_splits(axis_device device, const float *partial, float *out, int64_t len, int64_t splits,
+int sum_splits(axis_device device, const float *partial, float *out, int64_t len, int64_t stride, int64_t splits,
                const float *bias, int64_t n, const float *d, float alpha, float beta, int32_t perm_c,
                int32_t perm_taps, float *mid_space = nullptr, axis::Scratch *owner = nullptr) {
     const unsigned blocks = axis::blocks_for(len, 64, INT32_MAX);
     const bool defer = owner && device->deferring && len <= (int64_t)INT32_MAX * 64 / 2;
     auto last_pass = [&](const float *slices, int64_t count, axis::Scratch &held) {
         // four outputs per lane when every slice and the output start 16-byte aligned
-        const bool vec4 = len % 4 == 0 && axis::aligned16(slices) && axis::aligned16(out);
+        const bool vec4 = stride % 4 == 0 && axis::aligned16(slices) && axis::aligned16(out);
         if (defer) {
             axis::FinishTask t{};
             t.partial = slices;
@@ -821,7 +825,7 @@ int sum_splits(axis_device device, const float *partial, float *out, int64_t len
             t.d = d;
             t.len = len;
             t.count = count;
-            t.stride = len;
+            t.stride = stride;
             t.n = n;
             t.alpha = alpha;
             t.beta = beta;
@@ -833,10 +837,10 @@ int sum_splits(axis_device device, const float *partial, float *out, int64_t len
         }
         if (vec4) {
             split_sum4_kernel<<<axis::blocks_for(len, 256, INT32_MAX), 256, 0, device->stream>>>(
-                slices, out, len, (int32_t)count, len, bias, n, d, alpha, beta, perm_c, perm_taps);
+                slices, out, len, (int32_t)count, stride, bias, n, d, alpha, beta, perm_c, perm_taps);
             return axis::launch_status("split_sum4_kernel");
         }
-        split_sum_kernel<<<blocks, 256, 0, device->stream>>>(slices, out, len, (int32_t)count, len, bias, n, d,
+        split_sum_kernel<<<blocks, 256, 0, device->stream>>>(slices, out, len, (int32_t)count, stride, bias, n, d,
                                                              alpha, beta, perm_c, perm_taps);
         return axis::launch_status("split_sum_kernel");
     };
@@ -847,11 +851,11 @@ int sum_splits(axis_device device, const float *partial, float *out, int64_t len
     axis::Scratch mid;
     float *sums = mid_space;
     if (!sums || defer) {
-        if (int st = mid.get(device, sizeof(float) * (size_t)(ranges * len))) return st;
+        if (int st = mid.get(device, sizeof(float) * (size_t)(ranges * stride))) return st;
         sums = mid.as<float>();
     }
     dim3 grid(axis::blocks_for(len, 256, INT32_MAX), (unsigned)ranges);
-    split_range_kernel<<<grid, 256, 0, device->stream>>>(partial, sums, len, (int32_t)splits, span);
+    split_range_kernel<<<grid, 256, 0, device->stream>>>(partial, sums, len, stride, (int32_t)splits, span);
     if (int st = axis::launch_status("split_range_kernel")) return st;
     return last_pass(sums, ranges, mid);
 }
@@ -904,16 +908,16 @@ int run_gemm_bf16(axis_device device, const GemmParams &p, int64_t batch, float 
     g.k_chunk = chunk;
     g.splits = (int32_t)splits;
     if (splits > 1) {
-        if (int st = partial.get(device, sizeof(float) * (size_t)(out_len * splits))) return st;
+        if (int st = partial.get(device, sizeof(float) * (size_t)(slice_stride(out_len) * splits))) return st;
         g.c = partial.as<float>();
-        g.c_split = out_len;
+        g.c_split = slice_stride(out_len);
     } else {
         g.c = out;
         g.c_split = 0;
     }
     if (int st = axis::bf16_gemm(device, g, batch, tile)) return st;
     if (splits > 1)
-        return sum_splits(device, partial.as<float>(), out, out_len, splits, p.bias, p.n, p.d, p.alpha, p.beta, 0, 0);
+        return sum_splits(device, partial.as<float>(), out, out_len, slice_stride(out_len), splits, p.bias, p.n, p.d, p.alpha, p.beta, 0, 0);
     return AXIS_OK;
 }
 
@@ -1032,25 +1036,29 @@ int run_gemm(axis_device device, GemmParams p, int64_t batch, float *out, const 
     axis::Scratch partial, ordered;
     // spare: the range sums of more than 32 slices, or an unsplit permuted product before its move
     float *partials = nullptr, *spare = nullptr;
+    int64_t stride = slice_stride(out_len);
     if (ws) {
         const int64_t ranges = splits > 32 ? (splits + 31) / 32 : 0;
-        const int64_t need =
-            (splits > 1 && !fold ? splits + ranges : 0) * out_len + (splits == 1 && p.perm_c ? out_len : 0);
+        auto needed = [&]() {
+            return (splits > 1 && !fold ? splits + ranges : 0) * stride + (splits == 1 && p.perm_c ? out_len : 0);
+        };
+        if (needed() > ws->floats) stride = out_len;  // the last product that fits without the padding
+        const int64_t need = needed();
         if (need > ws->floats)
             return axis::fail(AXIS_ERROR_INVALID, "product needs " + std::to_string(need * 4) +
                                                       " bytes of partial sums; the static scratch holds " +
                                                       std::to_string(ws->floats * 4));
         partials = ws->ptr;
-        spare = ws->ptr + splits * out_len;
+        spare = ws->ptr + splits * stride;
     }
     if (splits > 1 && !fold) {
         if (!partials) {
-            int status = partial.get(device, sizeof(float) * (size_t)(out_len * splits));
+            int status = partial.get(device, sizeof(float) * (size_t)(stride * splits));
             if (status) return status;
             partials = partial.as<float>();
         }
         p.c = partials;
-        p.c_split = out_len;
+        p.c_split = stride;
         p.c_batch = p.m * p.n;
     } else {
         // an unsplit product with permuted rows is written in its own order, then moved
@@ -1106,7 +1114,7 @@ int run_gemm(axis_device device, GemmParams p, int64_t batch, float *out, const 
     if (!on_planes) status = axis::launch_status("gemm_kernel");
     if (status) return status;
     if (splits > 1 && !fold)
-        status = sum_splits(device, partials, out, out_len, splits, p.bias, p.n, p.d, p.alpha, p.beta,
+        status = sum_splits(device, partials, out, out_len, stride, splits, p.bias, p.n, p.d, p.alpha, p.beta,
                             p.perm_c, p.perm_taps, spare, final_out && !ws ? &partial : nullptr);
     else if (p.perm_c) {
         // mode 2 of the weight permutation with the taps as one axis

@@ -454,19 +454,28 @@ __device__ __forceinline__ void store_tile(const GemmParams &p, const floatx4 (&
                 }
         }
     } else {
+        // rows that start on any element: the same vector stores (global memory takes them on 4 bytes)
+        // where all FN columns are there, else one by one
+        typedef float vec __attribute__((ext_vector_type(FN), aligned(4)));
 #pragma unroll
-        for (int b = 0; b < FN; ++b) {
-            if (col + b >= p.n) continue;
+        for (int a = 0; a < FM; ++a)
 #pragma unroll
-            for (int a = 0; a < FM; ++a)
+            for (int v = 0; v < 4; ++v) {
+                const int64_t row = row0 + RS * v + a;
+                if (row >= p.m || col >= p.n) continue;
+                const int64_t idx = row * p.n + col;
+                vec o;
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int64_t row = row0 + RS * v + a;
-                    if (row < p.m)
-                        c[row * p.n + col + b] = finish_value(bias, d, p.alpha, p.beta, acc[a][b][v],
-                                                              out_base + row * p.n + col + b, col + b);
+                for (int b = 0; b < FN; ++b)
+                    o[b] = col + b < p.n ? finish_value(bias, d, p.alpha, p.beta, acc[a][b][v], out_base + idx + b, col + b) : 0.f;
+                if (col + FN <= p.n) {
+                    *reinterpret_cast<vec *>(c + idx) = o;
+                } else {
+#pragma unroll
+                    for (int b = 0; b < FN; ++b)
+                        if (col + b < p.n) c[idx + b] = o[b];
                 }
-        }
+            }
     }
 }
 
