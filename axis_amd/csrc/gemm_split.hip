@@ -20,7 +20,9 @@
 // whose operand lies wholly below 2^-63, where the low planes approach the end of the exponent
 // range) are found at the end of a block -- any such value leaves its accumulators non-finite, and
 // the staged exponents are or-ed as they pass -- and the block then computes its tile again with
-// the fp32 matrix instruction.
+// the fp32 matrix instruction.  In a block with ordinary magnitudes too, an element below 2^-110 (1e-33)
+// may lose what its low planes would hold below 2^-126, the smallest normal number: at most 2^-126 times
+// what it is multiplied with, which shows only where a whole row of sums is that small.
 #include <algorithm>
 
 #include "gemm_split.hpp"
@@ -256,7 +258,7 @@ struct PlaneDense : PlaneStaging<BT, NT, RCONTIG> {
 // XMODE: 0 dense X, 2 convolution cols mode, 3 cols mode over aligned pixel steps, 4 rows mode with tap
 // steps in block-major order, 5 rows mode with per-lane taps.  STAGES LDS stages of both operands' planes.
 template <int BM, int BN, int WM, int WN, int STAGES, int PF, bool XR, bool YR, bool AL, int XMODE>
-__global__ void __launch_bounds__(WM *WN * 64, BM / WM == 32 ? (PF == 4 ? 2 : 3) : 2) split_gemm_kernel(GemmParams p) {
+__global__ void __launch_bounds__(WM *WN * 64, BM / WM == 32 ? 3 : 2) split_gemm_kernel(GemmParams p) {
     constexpr int NT = WM * WN * 64;
     constexpr int TM = BM / WM, TN = BN / WN, FM = TM / 16, FN = TN / 16;
     static_assert((TM == 64 || TM == 32) && (TN == 64 || TN == 32), "waves of 64 or 32 rows and columns");
@@ -342,8 +344,8 @@ __global__ void __launch_bounds__(WM *WN * 64, BM / WM == 32 ? (PF == 4 ? 2 : 3)
     };
 
     // One staged step; in an odd one the first operand is staged negated and the chains subtracted (the
-    // instruction's roundings lean one way, see the top).  between(b): work placed with column block b's MFMAs (the next stage's splits and
-    // stores, the loads after them).
+    // instruction's roundings lean one way, see the top).  between(b): work placed with column block
+    // b's MFMAs (the next stage's splits and stores, the loads after them).
     // G column blocks run their chains together: four or more independent MFMAs per link of the chain
     // cover the instruction's latency.
     constexpr int G = FM == 2 ? 2 : 1;
@@ -581,10 +583,10 @@ SplitPlan split_plan(int64_t m, int64_t n, int64_t k, int64_t batch, int64_t cus
         const double ragged = aligned ? 1.0 : 1.2;
         const int64_t tiles = ((m + sh.rows - 1) / sh.rows) * ((n + sh.cols - 1) / sh.cols) * batch;
         const int64_t most = std::max<int64_t>(1, std::min<int64_t>(k / (2 * kDepth), 512));
-        for (int64_t want = 1; want <= most; ++want) {
-            int64_t chunk = (k + want - 1) / want;
-            chunk = (chunk + kDepth - 1) / kDepth * kDepth;
-            if ((k + chunk - 1) / chunk != want) continue;
+        // the least slice count of each slice length (most of 2 sqrt(k / 32) of them): 17 -> 6 us of host
+        // time at [2, 100000] x [100000, 2], together with the sums' bound below
+        for (int64_t want = 1, chunk; want <= most; want = (k + chunk - kDepth - 1) / (chunk - kDepth)) {
+            chunk = ((k + want - 1) / want + kDepth - 1) / kDepth * kDepth;
             // slices, and range sums of more than 32 of them, stay within 64 MiB
             if (want > 1 && (want + (want > 32 ? (want + 31) / 32 : 0)) * out_len > (int64_t(16) << 20)) break;
             const double us = ragged * launch_us(tiles * want, (double)(chunk / kDepth), sh.rate, cus) +
@@ -593,7 +595,9 @@ SplitPlan split_plan(int64_t m, int64_t n, int64_t k, int64_t batch, int64_t cus
                 best_us = us;
                 plan = {sh.tile, sh.rows, sh.cols, want};
             }
-            if (tiles * want > 8 * cus) break;  // more slices only add to the sum
+            // more slices only add to the sum
+            if (tiles * want > 8 * cus || sh.rate.round_us + slices_us(want, out_len) >= best_us) break;
+            if (chunk <= kDepth) break;
         }
     }
     return plan;

@@ -69,6 +69,22 @@ def test_magnitudes_at_the_ends_of_the_range(dev, m, k, n, sx, sy):
     assert np.all(np.abs(got - xd @ yd) <= bound(xd, yd, k))
 
 
+@pytest.mark.parametrize("m,k,n", [(2048, 512, 1024), (1030, 1001, 515)])
+def test_tiny_values_among_ordinary_ones(dev, m, k, n):
+    # rows (and single elements) of 1e-36 in tiles that keep the planes: what the low planes lose is below
+    # the smallest normal number per element of either operand
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    y = rng.standard_normal((k, n)).astype(np.float32)
+    x[::7] *= np.float32(1e-36)
+    x[:, ::5] *= np.float32(1e-34)
+    y[3::11, ::3] *= np.float32(1e-37)
+    xd, yd = x.astype(np.float64), y.astype(np.float64)
+    lost = 2.0 ** -126 * (np.abs(xd).sum(1)[:, None] + np.abs(yd).sum(0)[None, :])
+    got = run(dev, "axis_matmul", x, y, 1, m, k, n, m * n).reshape(m, n)
+    assert np.all(np.abs(got - xd @ yd) <= bound(xd, yd, k) + lost)
+
+
 @pytest.mark.parametrize("m,k,n", [(2048, 512, 1024), (1030, 1001, 515), (512, 4096, 512)])
 def test_values_the_planes_do_not_hold(dev, m, k, n):
     # infinities, NaN and magnitudes that bf16 rounds to infinity give what fp32 products give
